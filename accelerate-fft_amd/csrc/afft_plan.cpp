@@ -695,9 +695,41 @@ struct Builder {
             return n <= dev.max_lds_len[plan.dtype] && mixed_shape(plan.dtype, n, s_ * o, strided, false, dev.lds_bytes, 0, 0, sh)
                        ? AxisKind::kSingle : AxisKind::kBluestein;
         }
-        if (n > dev.max_lds_len[plan.dtype] || (strided && split_strided(n, s_))) return AxisKind::kSplit;
+        const int64_t limit = dev.max_lds_len[plan.dtype];
         MixShape sh;
-        return mixed_shape(plan.dtype, n, s_ * o, strided, false, dev.lds_bytes, 0, 0, sh) ? AxisKind::kSingle : AxisKind::kSplit;
+        if (n <= limit && !(strided && split_strided(n, s_)) &&
+            mixed_shape(plan.dtype, n, s_ * o, strided, false, dev.lds_bytes, 0, 0, sh))
+            return AxisKind::kSingle;
+        // (11^7, say, has no two factors of one workgroup each: chirp-z, whose padded length has)
+        int64_t n1, n2, m2;
+        const bool splits = is_5smooth(n) || (!strided && (six_step_n1(n) || split_six_step_factors(n, o, n1, n2, m2))) ||
+                            balanced_factors(n, n1, n2);
+        return splits ? AxisKind::kSplit : AxisKind::kBluestein;
+    }
+
+    // whether a strided axis of length n can be one launch (the lengths of the register kernel and of
+    // the compiled columns have a mixed-radix tile too)
+    bool strided_kernel(int64_t n)
+    {
+        MixShape sh;
+        return mixed_shape(plan.dtype, n, (int64_t)1 << 30, true, false, dev.lds_bytes, 0, 0, sh);
+    }
+
+    // The most balanced factors n = n1 * n2 of a four-step transform, n1 <= n2, both lengths of one
+    // strided launch; false if there are none.
+    bool balanced_factors(int64_t n, int64_t &n1, int64_t &n2)
+    {
+        const int64_t limit = dev.max_lds_len[plan.dtype];
+        int64_t d = (int64_t)std::sqrt((double)n);
+        while (d * d > n) --d;
+        for (; d >= 2 && n / d <= limit; --d) {
+            if (n % d || !is_13smooth(d) || !is_13smooth(n / d)) continue;
+            if (!strided_kernel(n / d) || !strided_kernel(d)) continue;
+            n1 = d;
+            n2 = n / d;
+            return true;
+        }
+        return false;
     }
 
     // two-level table for W_n^e: lo[e & (2^sh - 1)], hi[e >> sh]
@@ -876,7 +908,6 @@ struct Builder {
         a.st1 = 0;
         a.st2 = n * s_;
         a.es = s_;
-        const int64_t limit = dev.max_lds_len[plan.dtype];
         switch (axis_kind(n, s_, o)) {
         case AxisKind::kRows: add_rows(n, ntrans, src, cur, pick_row_variant(n, ntrans)); return cur;
         case AxisKind::kSingle: add_stockham(n, ntrans, a, a, strided, src, cur); return cur;
@@ -897,19 +928,7 @@ struct Builder {
         // balanced four-step (strided axes, and rows neither six-step form covers):
         // n = n1 * n2, element i = i1*n2 + i2, output k = k1 + n1*k2
         int64_t n1 = 0, n2 = 0;
-        double best = 1e300;
-        for (int64_t d = 2; d <= limit; ++d) {
-            if (n % d) continue;
-            const int64_t e = n / d;
-            if (e > limit || !is_13smooth(d) || !is_13smooth(e)) continue;
-            const double sc = std::fabs(std::log((double)d) - std::log((double)e));
-            if (sc < best) {
-                best = sc;
-                n1 = d;
-                n2 = e;
-            }
-        }
-        if (!n1) {
+        if (!balanced_factors(n, n1, n2)) {
             status = AFFT_ERROR_UNSUPPORTED_SIZE;
             return cur;
         }

@@ -1,0 +1,73 @@
+"""The planner on the host: plans are made and run against a stand-in for the HIP runtime
+(hip_host_stub.c, preloaded into a child process), which allocates from the heap and records the
+shape of every launch instead of running it."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+CHILD = """
+import ctypes, importlib.util
+spec = importlib.util.spec_from_file_location("_lib", {lib!r})
+L = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(L)
+lib = L.lib()
+stub = ctypes.CDLL(None)
+stub.stub_most_groups.restype = stub.stub_most_threads.restype = ctypes.c_ulonglong
+
+def plan(dtype, *ext, axes=L.AXES_INNERMOST):
+    h = ctypes.c_void_p()
+    return lib.afft_plan_create(ctypes.byref(h), dtype, len(ext), L.extents_arg(ext), axes, 0), h
+
+def largest_prime(n):
+    p, most = 2, 1
+    while p * p <= n:
+        while n % p == 0:
+            most, n = p, n // p
+        p += 1
+    return max(most, n) if n > 1 else most
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libhip_host_stub.so")
+    r = subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-w", "-I/opt/rocm/include",
+                        os.path.join(HERE, "hip_host_stub.c"), "-o", out], capture_output=True, text=True)
+    if r.returncode:
+        pytest.skip("no C compiler or HIP headers: " + r.stderr[-300:])
+    return out
+
+
+def run_child(stub, code):
+    head = CHILD.format(lib=os.path.join(ROOT, "accelerate-fft_amd", "afft", "_lib.py"))
+    r = subprocess.run([sys.executable, "-c", head + code], env=dict(os.environ, LD_PRELOAD=stub),
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+def test_every_long_smooth_length_has_a_plan(stub):
+    """Lengths beyond one workgroup with prime factors up to 13: two factors with kernels of their
+    own (the most balanced ones may have none: Complex Double 2 * 13^6 = 2197 * 4394 has no tile of
+    4394), or chirp-z where there are no such factors (Complex Double 11^7)."""
+    run_child(stub, """
+lo, hi = 1 << 22, 1 << 25
+lengths = {1}
+for p in (2, 3, 5, 7, 11, 13):
+    lengths |= {a * p ** k for a in lengths for k in range(1, 26) if a * p ** k <= hi}
+bad = []
+for n in sorted(lengths):
+    if n < lo or largest_prime(n) < 7:
+        continue
+    for dtype in (L.C64, L.C128):
+        st, h = plan(dtype, n)
+        if st:
+            bad.append((dtype, n, st))
+        else:
+            lib.afft_plan_destroy(h)
+assert not bad, (len(bad), bad[:10])
+""")
