@@ -56,6 +56,26 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, i
     return hipSuccess;
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
+/* the launch configuration between a call's <<<>>> and its stub */
+static dim3 cfg_grid, cfg_block;
+static size_t cfg_lds;
+static hipStream_t cfg_stream;
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t s)
+{
+    cfg_grid = grid;
+    cfg_block = block;
+    cfg_lds = lds;
+    cfg_stream = s;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipStream_t *s)
+{
+    *grid = cfg_grid;
+    *block = cfg_block;
+    *lds = cfg_lds;
+    *s = cfg_stream;
+    return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t lds, hipStream_t s)
 {
     (void)f; (void)args; (void)lds; (void)s;

@@ -71,3 +71,21 @@ for n in sorted(lengths):
             lib.afft_plan_destroy(h)
 assert not bad, (len(bad), bad[:10])
 """)
+
+
+def test_the_identity_copies_whole_tiles(stub):
+    """A transform over extents of 1 is a copy: at least 256 elements to a workgroup, and a grid of
+    fewer than 2^32 threads for arrays of 2^32 elements too."""
+    run_child(stub, """
+for dtype in (L.C64, L.C128):
+    for shape, axes in (((1000, 1), L.AXES_INNERMOST), (((1 << 24) + 3, 1), L.AXES_INNERMOST),
+                        (((1 << 32) + 3, 1), L.AXES_INNERMOST), ((1, 1), L.AXES_ALL)):
+        st, h = plan(dtype, *shape, axes=axes)
+        assert st == 0
+        stub.stub_reset()
+        assert lib.afft_exec(h, -1, 256, 512, 1.0, None) == 0  # (no kernel reads these addresses)
+        groups, threads = stub.stub_most_groups(), stub.stub_most_threads()
+        assert 1 <= groups <= max(1024, shape[0] // 256 + 1), (dtype, shape, groups)
+        assert threads < 1 << 32
+        lib.afft_plan_destroy(h)
+""")
