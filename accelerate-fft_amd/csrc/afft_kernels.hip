@@ -12,6 +12,7 @@
 
 #include "afft_device.hpp"
 #include "afft_internal.hpp"
+#include "afft_mixed.hpp"
 
 namespace afft {
 
@@ -156,6 +157,19 @@ __global__ void afft_gen_pass_twiddles(typename cplx_of<Real>::type *out, const 
 }
 
 template <typename Real>
+__global__ void afft_gen_mixed_twiddles(typename cplx_of<Real>::type *out, int Ns, int R)
+{
+    using V = typename cplx_of<Real>::type;
+    const int count = mixed_twiddle_elems(sizeof(Real) == 8, Ns, R);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (R + 1) * Ns; i += gridDim.x * blockDim.x) {
+        const int r = i / Ns + 1, k = i % Ns, at = mixed_twiddle_at(sizeof(Real) == 8, Ns, r, k);
+        double s, co;
+        sincospi(-2.0 * (double)(r * k) / (double)(Ns * R), &s, &co); // (r k < 2^31, exact)
+        if (at < count) out[at] = c_make<V>((Real)co, (Real)s);       // (r = R fills the spare halves)
+    }
+}
+
+template <typename Real>
 __global__ void afft_gen_power_table(typename cplx_of<Real>::type *out, int64_t L, int64_t step,
                                      int64_t count)
 {
@@ -295,6 +309,19 @@ hipError_t gen_pass_twiddles(int dtype, void *out, const PassTable &pt, hipStrea
         hipLaunchKernelGGL(afft_gen_pass_twiddles<float>, dim3(g), dim3(256), 0, s, (float2 *)out, pt);
     else
         hipLaunchKernelGGL(afft_gen_pass_twiddles<double>, dim3(g), dim3(256), 0, s, (double2 *)out, pt);
+    return hipGetLastError();
+}
+
+hipError_t gen_mixed_twiddles(int dtype, void *out, const MixArgs &a, hipStream_t s)
+{
+    for (int i = 1; i < a.npass; ++i) {
+        const MixPass &p = a.pass[i];
+        const int64_t g = gs_grid((int64_t)p.Ns * (p.R + 1));
+        if (dtype == 0)
+            hipLaunchKernelGGL(afft_gen_mixed_twiddles<float>, dim3(g), dim3(256), 0, s, (float2 *)out + p.toff, p.Ns, p.R);
+        else
+            hipLaunchKernelGGL(afft_gen_mixed_twiddles<double>, dim3(g), dim3(256), 0, s, (double2 *)out + p.toff, p.Ns, p.R);
+    }
     return hipGetLastError();
 }
 

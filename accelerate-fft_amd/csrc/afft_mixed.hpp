@@ -32,7 +32,7 @@ __host__ __device__ constexpr int mixed_butterflies(int E, int R)
 // One pass: butterflies of radix R at stride Ns, nb = n / R of them per transform.
 struct MixPass {
     int R, Ns, nb;
-    int step;          // n / (Ns R): the pass's twiddle W_{Ns R}^k is W_n^{k step}
+    int toff;          // elements in front of the pass's twiddles in MixArgs::tw
     uint32_t mnb, mns; // floor(2^32 / d) + 1 for d = nb and d = Ns (unused for d = 1)
     // LDS layouts, in elements: the pass reads block q of Ns elements rpad q elements on, its
     // butterflies' elements rstep apart, and writes its own blocks of Ns R elements wblock apart
@@ -50,10 +50,22 @@ __host__ __device__ constexpr int mixed_waves(bool f64, int E, bool rows, bool c
     return chirpz ? 4 : rows ? 6 : 5;
 }
 
+// Where the table of a pass holds W_{Ns R}^{r k}, r = 1 ... R - 1, k < Ns, in elements from its start:
+// neighbouring lanes have neighbouring k, and 16 bytes hold the Complex Float powers 2p + 1 and 2p + 2.
+__host__ __device__ constexpr int mixed_twiddle_at(bool f64, int Ns, int r, int k)
+{
+    return f64 ? (r - 1) * Ns + k : 2 * ((r - 1) / 2 * Ns + k) + (r - 1) % 2;
+}
+__host__ __device__ constexpr int mixed_twiddle_elems(bool f64, int Ns, int R)
+{
+    return f64 ? (R - 1) * Ns : 2 * (R / 2) * Ns;
+}
+
 struct MixArgs {
     const void *in;
     void *out;
-    const void *tw;    // W_n^m, m in [0, n)
+    const void *tw;    // the passes' twiddles (mixed_twiddle_at)
+    int tw_elems;
     int64_t ntrans;
     Addr ain, aout;
     AddrDiv div;       // of a transform index by ain.cnt0 and ain.cnt1 (= aout's)
@@ -77,6 +89,91 @@ struct MixArgs {
     const void *post_hi, *post_lo;
     // chirp-z: c[m], m < len, and the filter of n elements
     const void *chirp, *filt;
+};
+
+// The twiddles of one butterfly of a pass: W_{Ns R}^{r k}, r = 1 ... R - 1, read from the pass's table, B
+// of them with the butterfly's elements (load) and the others B at a time (apply).  B = 0: the powers 1, 2, 3,
+// 4, 8 and 12, and the others as one product of two of them; a prime radix beyond 16: the powers 1, 2,
+// 4, 8 and 16, and the others as their products.
+template <int R, typename V, int B> struct MixTwiddles {
+    static constexpr bool f64 = sizeof(V) == 16;
+    static constexpr int S = (int)sizeof(V);
+    static constexpr int N = R > 16 ? 5 : B == 0 ? 6 : (B < R ? B : R);
+    static_assert(B % 2 == 0, "whole loads");
+    V w[N];
+    __device__ __forceinline__ static uint32_t base(const MixPass &P, int k)
+    {
+        return (uint32_t)((P.toff + (f64 ? k : 2 * k)) * S);
+    }
+    __device__ __forceinline__ static void one(V &to, const BufView &tw, const MixPass &P, uint32_t off, int r)
+    {
+        to = buf_load<V>(tw, off, (uint32_t)(mixed_twiddle_at(f64, P.Ns, r, 0) * S));
+    }
+    // powers r and r + 1, r odd
+    __device__ __forceinline__ static void two(V &a, V &b, const BufView &tw, const MixPass &P, uint32_t off, int r)
+    {
+        if constexpr (f64) {
+            one(a, tw, P, off, r);
+            if (r + 1 < R) one(b, tw, P, off, r + 1);
+        } else {
+            const float4 q = buf_load<float4>(tw, off, (uint32_t)((r - 1) / 2 * P.Ns * 16));
+            a = c_make<V>(q.x, q.y);
+            b = c_make<V>(q.z, q.w);
+        }
+    }
+    // the powers from r0 on, as many as fit
+    __device__ __forceinline__ void batch(const BufView &tw, const MixPass &P, uint32_t off, int r0)
+    {
+#pragma unroll
+        for (int u = 0; u < N && r0 + u < R; u += 2) {
+            if (u + 1 < N) two(w[u], w[u + 1], tw, P, off, r0 + u);
+            else one(w[u], tw, P, off, r0 + u);
+        }
+    }
+    __device__ __forceinline__ void load(const BufView &tw, const MixPass &P, int k)
+    {
+        const uint32_t off = base(P, k);
+        if constexpr (R > 16) {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) one(w[q], tw, P, off, 1 << q);
+        } else if constexpr (B > 0) {
+            batch(tw, P, off, 1);
+        } else {
+            if constexpr (R > 2) two(w[0], w[1], tw, P, off, 1);
+            else one(w[0], tw, P, off, 1);
+            if constexpr (R > 4) two(w[2], w[3], tw, P, off, 3);
+            else if constexpr (R > 3) one(w[2], tw, P, off, 3);
+            if constexpr (R > 8) one(w[4], tw, P, off, 8);
+            if constexpr (R > 12) one(w[5], tw, P, off, 12);
+        }
+    }
+    __device__ __forceinline__ void apply(V *v, const BufView &tw, const MixPass &P, int k)
+    {
+        if constexpr (R > 16) {
+            power_twiddles<R>(v, w);
+        } else if constexpr (B > 0) {
+#pragma unroll
+            for (int r0 = 1; r0 < R; r0 += N) {
+                if (r0 > 1) {
+                    __builtin_amdgcn_sched_barrier(0); // (registers)
+                    batch(tw, P, base(P, k), r0);
+                }
+#pragma unroll
+                for (int u = 0; u < N && r0 + u < R; ++u) v[r0 + u] = c_mul(v[r0 + u], w[u]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                const int g = r & 12, m = r & 3;
+                if (g == 0) {
+                    v[r] = c_mul(v[r], w[m - 1]);
+                } else {
+                    const V &q = w[g == 4 ? 3 : g == 8 ? 4 : 5];
+                    v[r] = c_mul(v[r], m ? c_mul(q, w[m - 1]) : q);
+                }
+            }
+        }
+    }
 };
 
 // Host-side shape of a launch (afft_mixed_plan.cpp).
@@ -113,7 +210,9 @@ bool mixed_tile(int dtype, int64_t n, bool chirpz, int block, int elems, MixShap
 // padded length of a chirp-z transform of n points in such a tile, 0 if none fits
 int64_t mixed_chirpz_tile(int64_t n, int block, int elems);
 
-void mixed_fill(const MixShape &sh, int64_t n, MixArgs &a);
+void mixed_fill(int dtype, const MixShape &sh, int64_t n, MixArgs &a);
+// The twiddle table of a's passes (tw_elems elements), in FP64 and rounded.
+hipError_t gen_mixed_twiddles(int dtype, void *out, const MixArgs &a, hipStream_t s);
 
 hipError_t launch_mixed(int dtype, const MixArgs &a, bool strided, int E, int block, int64_t grid, size_t lds,
                         hipStream_t s);

@@ -356,8 +356,8 @@ struct Builder {
         l.E = sh.E;
         MixArgs &a = l.ma;
         if (chirpz && !bluestein_tables(len, n, a.chirp, a.filt)) return;
-        a.tw = power_table(n);
-        if (status) return;
+        mixed_fill(plan.dtype, sh, n, a);
+        if (!mixed_table(a)) return;
         a.ntrans = ntrans;
         a.ain = ain;
         a.aout = aout;
@@ -365,7 +365,6 @@ struct Builder {
         a.len = (int)len;
         a.odd_in = (int)(ain.es / axis_stride) & 1;
         a.odd_out = (int)(aout.es / axis_stride) & 1;
-        mixed_fill(sh, n, a);
         a.xcd_remap = strided && !getenv_flag("AFFT_NO_XCD") ? 1 : 0;
         a.scale = 1.0;
         a.post_L = post_L;
@@ -561,6 +560,22 @@ struct Builder {
         check(gen_power_table(plan.dtype, buf, n, 1, n, s));
         plan.pow_cache[n] = buf;
         return buf;
+    }
+
+    // the twiddles of a mixed-radix transform's passes, cached per sequence of radices
+    bool mixed_table(MixArgs &a)
+    {
+        std::vector<int> key;
+        for (int i = 0; i < a.npass; ++i) key.push_back(a.pass[i].R);
+        auto it = plan.mix_cache.find(key);
+        if (it == plan.mix_cache.end()) {
+            void *buf = alloc(std::max(1, a.tw_elems) * (int64_t)esz());
+            if (!buf) return false;
+            check(gen_mixed_twiddles(plan.dtype, buf, a, s));
+            it = plan.mix_cache.emplace(key, buf).first;
+        }
+        a.tw = it->second;
+        return status == AFFT_SUCCESS;
     }
 
     // Persistent row kernel (compiled layout for this n).
@@ -932,16 +947,9 @@ struct Builder {
             status = AFFT_ERROR_UNSUPPORTED_SIZE;
             return cur;
         }
-        // two-level table for W_n^e: lo[e & (2^sh - 1)], hi[e >> sh]
+        const void *hi = nullptr, *lo = nullptr;
         int sh = 0;
-        while (((int64_t)1 << (2 * sh)) < n) ++sh;
-        const int64_t lo_cnt = (int64_t)1 << sh;
-        const int64_t hi_cnt = (n + lo_cnt - 1) / lo_cnt;
-        void *lo = alloc(lo_cnt * (int64_t)esz());
-        void *hi = alloc(hi_cnt * (int64_t)esz());
-        if (status) return cur;
-        check(gen_power_table(plan.dtype, lo, n, 1, lo_cnt, s));
-        check(gen_power_table(plan.dtype, hi, n, lo_cnt, hi_cnt, s));
+        if (!power_tables(n, hi, lo, sh)) return cur;
         const Slot next = other(cur);
         int64_t &room = next == Slot::kWork ? plan.work_elems
                         : next == Slot::kAux2 ? plan.aux2_elems : plan.aux_elems;
@@ -1061,6 +1069,7 @@ void free_plan(Plan &plan)
     plan.launches.clear();
     plan.tw_cache.clear();
     plan.pow_cache.clear();
+    plan.mix_cache.clear();
     plan.blue_cache.clear();
     if (plan.pool) plan.pool->clear(free_block);
 }
@@ -1397,13 +1406,10 @@ int table_pass_twiddles(Plan &owner, const DeviceInfo &dev, hipStream_t s, int64
     return b.status;
 }
 
-int table_power(Plan &owner, const DeviceInfo &dev, hipStream_t s, int64_t L, int64_t step,
-                int64_t count, const void *&out)
+int table_mixed(Plan &owner, const DeviceInfo &dev, hipStream_t s, MixArgs &a)
 {
     Builder b{owner, dev, s};
-    void *buf = b.alloc(count * (int64_t)b.esz());
-    if (!b.status) b.check(gen_power_table(owner.dtype, buf, L, step, count, s));
-    out = buf;
+    b.mixed_table(a);
     return b.status;
 }
 

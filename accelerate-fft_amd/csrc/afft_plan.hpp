@@ -74,6 +74,7 @@ struct Plan {
     int64_t device_bytes = 0;
     std::map<int64_t, const void *> tw_cache;
     std::map<int64_t, const void *> pow_cache;
+    std::map<std::vector<int>, const void *> mix_cache; // by radices
     std::map<std::pair<int64_t, int64_t>, std::pair<const void *, const void *>> blue_cache; // by (n, M)
     // elements of each per-execution array (0: the plan needs none of it)
     int64_t work_elems = 0;
@@ -119,8 +120,7 @@ void clear_cache();
 void *plan_alloc(Plan &owner, const DeviceInfo &dev, int64_t bytes, int &status);
 int table_pass_twiddles(Plan &owner, const DeviceInfo &dev, hipStream_t s, int64_t n,
                         const LdsLayout &L, PassTable &pt, const void *&tw);
-int table_power(Plan &owner, const DeviceInfo &dev, hipStream_t s, int64_t L, int64_t step,
-                int64_t count, const void *&out);
+int table_mixed(Plan &owner, const DeviceInfo &dev, hipStream_t s, MixArgs &a);
 int table_bluestein(Plan &owner, const DeviceInfo &dev, hipStream_t s, int64_t n, int64_t M,
                     const void *&chirp, const void *&filt);
 bool is_5smooth(int64_t n);

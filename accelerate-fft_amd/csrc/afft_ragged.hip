@@ -33,7 +33,7 @@ __device__ __forceinline__ void run_item(const RaggedArgs &a, const RaggedClass 
     V *__restrict__ out = reinterpret_cast<V *>(a.out);
     const int64_t *__restrict__ moffs = a.moffs + first;
     const Real sc = a.inverse ? (Real)(1.0 / (double)len) : (Real)1, sy = a.conj ? -sc : sc;
-    const BufView vtw(reinterpret_cast<const V *>(K.m.tw), (uint32_t)(n * S));
+    const BufView vtw(reinterpret_cast<const V *>(K.m.tw), (uint32_t)(K.m.tw_elems * S));
     const BufView vchirp(reinterpret_cast<const V *>(K.m.chirp), (uint32_t)(len * S));
     const BufView vfilt(reinterpret_cast<const V *>(K.m.filt), (uint32_t)(n * S));
     const int npass = K.m.npass, pitch = K.m.pitch;
@@ -72,7 +72,8 @@ __device__ __forceinline__ void run_item(const RaggedArgs &a, const RaggedClass 
         auto body = [&](auto rc) __attribute__((always_inline)) {
             constexpr int R = decltype(rc)::value;
             constexpr int NK = mixed_butterflies(EMAX, R);
-            V v[NK][R], w[NK][4];
+            V v[NK][R];
+            MixTwiddles<R, V, S == 16 ? 6 : 16> w[NK];
             int cc[NK], cb[NK], cq[NK];
             bool ca[NK];
 #pragma unroll
@@ -82,13 +83,7 @@ __device__ __forceinline__ void run_item(const RaggedArgs &a, const RaggedClass 
                 cb[kk] = g - cc[kk] * P.nb;
                 ca[kk] = cc[kk] < count;
                 cq[kk] = mix_div(cb[kk], P.Ns, P.mns);
-                if (P.Ns > 1 && ca[kk]) {
-                    const uint32_t e = (uint32_t)((cb[kk] - cq[kk] * P.Ns) * P.step * S);
-                    w[kk][0] = buf_load<V>(vtw, e, 0);
-                    if constexpr (R > 2) w[kk][1] = buf_load<V>(vtw, 2 * e, 0);
-                    if constexpr (R > 4) w[kk][2] = buf_load<V>(vtw, 4 * e, 0);
-                    if constexpr (R > 8) w[kk][3] = buf_load<V>(vtw, 8 * e, 0);
-                }
+                if (P.Ns > 1 && ca[kk]) w[kk].load(vtw, P, cb[kk] - cq[kk] * P.Ns);
             }
             if (from_global) {
 #pragma unroll
@@ -128,7 +123,7 @@ __device__ __forceinline__ void run_item(const RaggedArgs &a, const RaggedClass 
             }
             if (P.Ns > 1) {
 #pragma unroll
-                for (int kk = 0; kk < NK; ++kk) power_twiddles<R>(v[kk], w[kk]);
+                for (int kk = 0; kk < NK; ++kk) w[kk].apply(v[kk], vtw, P, cb[kk] - cq[kk] * P.Ns);
             }
 #pragma unroll
             for (int kk = 0; kk < NK; ++kk) dft<R>::run(v[kk]);

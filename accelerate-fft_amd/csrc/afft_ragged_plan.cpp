@@ -122,11 +122,11 @@ struct Builder {
             const int64_t n = L > elems ? 0 : chirpz ? mixed_chirpz_tile(L, kRaggedBlock[rp.dtype][bin], elems) : L;
             MixShape sh;
             if (n < 1 || !class_tile(L, n, chirpz, rp.dtype, bin, rp.device, dev.lds_bytes, sh)) continue;
-            mixed_fill(sh, n, K.m);
+            mixed_fill(rp.dtype, sh, n, K.m);
             K.m.len = (int)L;
             C = sh.C;
             lds_need[bin] = std::max(lds_need[bin], sh.lds);
-            if (n > 1) status = table_power(rp.tables, dev, s, n, 1, n, K.m.tw);
+            if (n > 1) status = table_mixed(rp.tables, dev, s, K.m);
             if (!status && chirpz) status = table_bluestein(rp.tables, dev, s, L, n, K.m.chirp, K.m.filt);
             return !status;
         }
