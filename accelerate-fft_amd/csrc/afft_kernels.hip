@@ -137,6 +137,23 @@ __global__ void __launch_bounds__(256) afft_chirp(const ChirpArgs a)
 // ----------------------------------------------------------------------------------------------
 // Twiddle / chirp generation in FP64.
 
+// exp(-2 pi i e / L), 0 <= e < L < 2^60: reduced to an eighth of a turn in integers, since the rounding of e / L itself
+// would turn an angle near 2 pi by more than the result's rounding
+__device__ __forceinline__ double2 unit_root(int64_t e, int64_t L)
+{
+    const int64_t o = 8 * e / L, f = o & 1 ? (o + 1) * L - 8 * e : 8 * e - o * L; // from the nearest quarter turn
+    double s, c;
+    sincospi((double)f / (4.0 * (double)L), &s, &c);
+    if (f == L) s = c; // (the eighth itself: sinpi(1/4) comes out one unit low)
+    if (o & 1) s = -s;
+    switch ((o + 1) >> 1 & 3) {
+    case 0: return make_double2(c, -s);
+    case 1: return make_double2(-s, -c);
+    case 2: return make_double2(-c, s);
+    default: return make_double2(s, c);
+    }
+}
+
 template <typename Real>
 __global__ void afft_gen_pass_twiddles(typename cplx_of<Real>::type *out, const PassTable pt)
 {
@@ -148,9 +165,8 @@ __global__ void afft_gen_pass_twiddles(typename cplx_of<Real>::type *out, const 
         for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < L; idx += gridDim.x * blockDim.x) {
             const int k = idx / R, r = idx % R;
             const int e = r * k; // < L, exact
-            double s, co;
-            sincospi(-2.0 * (double)e / (double)L, &s, &co);
-            out[pt.tw_off[p] + idx] = c_make<V>((Real)co, (Real)s);
+            const double2 w = unit_root(e, L);
+            out[pt.tw_off[p] + idx] = c_make<V>((Real)w.x, (Real)w.y);
         }
         Ns = L;
     }
@@ -163,9 +179,8 @@ __global__ void afft_gen_mixed_twiddles(typename cplx_of<Real>::type *out, int N
     const int count = mixed_twiddle_elems(sizeof(Real) == 8, Ns, R);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (R + 1) * Ns; i += gridDim.x * blockDim.x) {
         const int r = i / Ns + 1, k = i % Ns, at = mixed_twiddle_at(sizeof(Real) == 8, Ns, r, k);
-        double s, co;
-        sincospi(-2.0 * (double)(r * k) / (double)(Ns * R), &s, &co); // (r k < 2^31, exact)
-        if (at < count) out[at] = c_make<V>((Real)co, (Real)s);       // (r = R fills the spare halves)
+        const double2 w = unit_root(r == R ? 0 : r * k, Ns * R); // (r k < Ns R < 2^31; r = R: the spare halves)
+        if (at < count) out[at] = c_make<V>((Real)w.x, (Real)w.y);
     }
 }
 
@@ -178,9 +193,8 @@ __global__ void afft_gen_power_table(typename cplx_of<Real>::type *out, int64_t 
          i += (int64_t)gridDim.x * blockDim.x) {
         // exponent reduced exactly in integers; i*step < 2^62 for every table built here
         const int64_t e = (i * step) % L;
-        double s, co;
-        sincospi(-2.0 * (double)e / (double)L, &s, &co);
-        out[i] = c_make<V>((Real)co, (Real)s);
+        const double2 w = unit_root(e, L);
+        out[i] = c_make<V>((Real)w.x, (Real)w.y);
     }
 }
 
@@ -192,9 +206,8 @@ __global__ void afft_gen_twiddle_grid(typename cplx_of<Real>::type *out, int64_t
          i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t q = i / cols, j = i - q * cols;
         const int64_t e = (q * j) % L;
-        double s, co;
-        sincospi(-2.0 * (double)e / (double)L, &s, &co);
-        out[i] = c_make<V>((Real)co, (Real)s);
+        const double2 w = unit_root(e, L);
+        out[i] = c_make<V>((Real)w.x, (Real)w.y);
     }
 }
 
@@ -205,9 +218,8 @@ __global__ void afft_gen_chirp(typename cplx_of<Real>::type *out, int64_t n)
     for (int64_t m = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; m < n;
          m += (int64_t)gridDim.x * blockDim.x) {
         const int64_t e = (m * m) % (2 * n); // exp(-i pi m^2/n) has period 2n in m^2
-        double s, co;
-        sincospi(-(double)e / (double)n, &s, &co);
-        out[m] = c_make<V>((Real)co, (Real)s);
+        const double2 w = unit_root(e, 2 * n);
+        out[m] = c_make<V>((Real)w.x, (Real)w.y);
     }
 }
 
@@ -221,9 +233,8 @@ __global__ void afft_gen_bluestein_kernel(double2 *out, int64_t n, int64_t M)
         double2 v = make_double2(0.0, 0.0);
         if (src >= 0) {
             const int64_t e = (src * src) % (2 * n);
-            double s, co;
-            sincospi(-(double)e / (double)n, &s, &co);
-            v = make_double2(co, -s); // conj(chirp)
+            const double2 w = unit_root(e, 2 * n);
+            v = make_double2(w.x, -w.y); // conj(chirp)
         }
         out[m] = v;
     }

@@ -18,6 +18,10 @@ CASES = [
     (torch.complex64, 519, 1009, 1.78e-7),
     (torch.complex64, 8, 120000, 1.53e-7),     # two strided passes
     (torch.complex128, 1, 262144, 2.89e-16),
+    # chirp-z, whose tables hold angles that are no binary fractions of a turn
+    (torch.complex128, 64, 1009, 5.04e-16),
+    (torch.complex128, 83, 783, 4.59e-16),
+    (torch.complex128, 19, 3428, 4.83e-16),
 ]
 
 
