@@ -200,15 +200,16 @@ bool mixed_radices(int64_t n, bool symmetric, int E, int threads, MixShape &out,
 // False if it does not fit a workgroup.
 bool mixed_shape(int dtype, int64_t n, int64_t ntrans, bool strided, bool chirpz, size_t lds_bytes, int cus,
                  int cols, MixShape &out, bool gathered = false, bool layout = true);
-// The padded length of a chirp-z transform of length n: at least 2n - 1, the cheapest that fits
-// `limit` elements; 0 if none.
+int64_t bluestein_length(int64_t n);
+// The padded length of a chirp-z transform of length n: the cheapest of at least 2n - 1 that fits `limit`
+// elements and rounds no more than the lengths before it did; 0 if none.
 int64_t mixed_chirpz_length(int dtype, int64_t n, int64_t limit, size_t lds_bytes);
 // The shape of a tile of rows of length n for workgroups of `block` threads with 16 elements each, of at
 // most `elems` elements (the items of ragged batches): as many rows as fit.  False if none does.
 bool mixed_tile(int dtype, int64_t n, bool chirpz, int block, int elems, MixShape &out);
 
 // padded length of a chirp-z transform of n points in such a tile, 0 if none fits
-int64_t mixed_chirpz_tile(int64_t n, int block, int elems);
+int64_t mixed_chirpz_tile(int dtype, int64_t n, int block, int elems);
 
 void mixed_fill(int dtype, const MixShape &sh, int64_t n, MixArgs &a);
 // The twiddle table of a's passes (tw_elems elements), in FP64 and rounded.

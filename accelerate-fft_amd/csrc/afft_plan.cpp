@@ -158,19 +158,6 @@ bool choose_layout(int64_t n, int dtype, LdsLayout &out, int maxE, int maxT)
     return found;
 }
 
-// Bluestein padded length: the smallest M >= 2n - 1 of the form 2^k, 3*2^k or 5*2^k.
-int64_t bluestein_length(int64_t n)
-{
-    const int64_t need = 2 * n - 1;
-    int64_t best = 0;
-    for (int64_t base : {1, 3, 5}) {
-        int64_t m = base;
-        while (m < need) m *= 2;
-        if (best == 0 || m < best) best = m;
-    }
-    return best;
-}
-
 static PassTable make_pass_table(int64_t n, const LdsLayout &L, int64_t *tw_elems)
 {
     PassTable pt{};

@@ -91,7 +91,6 @@ Workspace carve_workspace(const Plan &plan, void *base);
 // Single-workgroup layout of length n: fewest passes, then E closest to 16; optional limits on
 // elements per thread and threads per transform.
 bool choose_layout(int64_t n, int dtype, LdsLayout &out, int maxE = 1 << 30, int maxT = -1);
-int64_t bluestein_length(int64_t n);
 int64_t lds_limit_elems(int dtype, size_t lds_bytes);
 int device_info(int device, DeviceInfo &out);
 int build_plan(Plan &plan, int dtype, int rank, const int64_t *extents, int axes, int device,

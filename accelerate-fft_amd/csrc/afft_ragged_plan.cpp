@@ -119,7 +119,7 @@ struct Builder {
         const bool chirpz = !is_13smooth(L);
         for (bin = 0; bin < (count < dev.cus ? 2 : 1); ++bin) {
             const int elems = kRaggedElems[rp.dtype][bin];
-            const int64_t n = L > elems ? 0 : chirpz ? mixed_chirpz_tile(L, kRaggedBlock[rp.dtype][bin], elems) : L;
+            const int64_t n = L > elems ? 0 : chirpz ? mixed_chirpz_tile(rp.dtype, L, kRaggedBlock[rp.dtype][bin], elems) : L;
             MixShape sh;
             if (n < 1 || !class_tile(L, n, chirpz, rp.dtype, bin, rp.device, dev.lds_bytes, sh)) continue;
             mixed_fill(rp.dtype, sh, n, K.m);

@@ -22,6 +22,11 @@ CASES = [
     (torch.complex128, 64, 1009, 5.04e-16),
     (torch.complex128, 83, 783, 4.59e-16),
     (torch.complex128, 19, 3428, 4.83e-16),
+    # chirp-z with a choice of padded lengths
+    (torch.complex64, 12787, 41, 1.31e-7),
+    (torch.complex64, 495, 1059, 1.62e-7),
+    (torch.complex64, 240, 2177, 1.71e-7),
+    (torch.complex128, 79, 824, 4.71e-16),
 ]
 
 
