@@ -151,14 +151,23 @@ afft_rows(const RowArgs a)
     // Five or more passes of the split exchange take four bases (W^k ... W^8k) a pass: the longer
     // products of two raised the error of 32768 points from 1.66e-7 to 1.85e-7.  16384 keeps two (same
     // error as with its former kernel; four: 1.46e-7, but 64 instead of 58 us for 1024 rows), and so do
-    // 16 Complex Double a thread, which would spill (3.9e-16 against 4.2e-16 in two passes).
-    constexpr bool kBases4 = SPLIT && NP > 4 && (sizeof(Real) == 4 || E < 16);
+    // 16 Complex Double a thread, which would spill (3.9e-16 against 4.2e-16 in two passes).  8 Complex Double
+    // a thread leave room for every twiddle of a pass (8192 points: 2.59e-16 with four bases, 2.41e-16).
+    constexpr bool kAll = SPLIT && sizeof(Real) == 8 && E <= 8;
+    constexpr bool kBases4 = SPLIT && !kAll && NP > 4 && (sizeof(Real) == 4 || E < 16);
     // base twiddles of pass p for thread index th; jb: of butterfly jb, where they differ
     auto base_twiddles = [&](auto pc, int th, V *w) {
         constexpr int p = decltype(pc)::value;
         constexpr int R = RL::R[p];
         constexpr int Ns = RL::ns(p);
-        if constexpr (Ns > 1) {
+        if constexpr (Ns > 1 && kAll) {
+            constexpr int SETS = T % Ns == 0 ? 1 : E / R;
+            constexpr int STEP = N / (Ns * R);
+#pragma unroll
+            for (int jb = 0; jb < SETS; ++jb)
+#pragma unroll
+                for (int r = 1; r < R; ++r) w[jb * (R - 1) + r - 1] = tw[r * ((th + jb * T) % Ns) * STEP];
+        } else if constexpr (Ns > 1) {
             constexpr int B = E / R;
             // the last pass (Ns * R == N) has k = t + j*T exactly: one base W^t per thread, the
             // factor W^{jT} of butterfly j is a compile-time constant
@@ -235,7 +244,11 @@ afft_rows(const RowArgs a)
 #pragma unroll
                 for (int r = 0; r < R; ++r) v[r] = reg[j + r * B];
                 if constexpr (Ns > 1) {
-                    if constexpr (kBases4) {
+                    if constexpr (kAll) {
+                        constexpr int first = T % Ns == 0 ? 0 : j * (R - 1);
+#pragma unroll
+                        for (int r = 1; r < R; ++r) v[r] = c_mul(v[r], tb[p][first + r - 1]);
+                    } else if constexpr (kBases4) {
                         constexpr int jt = T % Ns == 0 ? 0 : j * T;
                         const V w[4] = {twiddle_const<N, jt>(tb[p][0]), twiddle_const<N, 2 * jt>(tb[p][1]),
                                         twiddle_const<N, 4 * jt>(tb[p][2]), twiddle_const<N, 8 * jt>(tb[p][3])};

@@ -27,6 +27,8 @@ CASES = [
     (torch.complex64, 495, 1059, 1.62e-7),
     (torch.complex64, 240, 2177, 1.71e-7),
     (torch.complex128, 79, 824, 4.71e-16),
+    # rows through the split exchange
+    (torch.complex128, 260, 8192, 2.36e-16),
 ]
 
 
