@@ -268,6 +268,14 @@ struct Builder {
         return C;
     }
 
+    // whether the single-pass tile of a strided axis reads whole lines
+    bool whole_lines(int64_t n, int64_t stride)
+    {
+        MixShape sh;
+        return mixed_shape(plan.dtype, n, stride, true, false, dev.lds_bytes, 0, 0, sh) &&
+               (int64_t)sh.C * (int64_t)esz() >= 128;
+    }
+
     // A strided axis whose single-pass tile would read row segments shorter than 64 bytes is split
     // into two passes (four-step) whose tiles read longer ones.  64-byte segments in one pass beat two
     // passes of whole lines (2048^2 Complex Double 82 -> 62 us, 2048 x 16384 Complex Float 299 -> 260
@@ -803,8 +811,8 @@ struct Builder {
     }
 
     // Factors of o contiguous rows n = n1 * m1 * m2 for a six-step whose rows n2 = m1 * m2 have
-    // no compiled row kernel: a register column length n1, a strided single-pass length m1 whose
-    // tiles read whole lines, and a row length m2 with a transposed-store form.  The register
+    // no compiled row kernel: a register column length n1, a strided single-pass length m1, and a row
+    // length m2 with a transposed-store form.  The register
     // pass runs one thread per column, o * n / n1 threads, and hides its load latency only with
     // about 8 waves per CU: the longest n1 that keeps that many, else the shortest.  False if none.
     bool split_six_step_factors(int64_t n, int64_t o, int64_t &n1, int64_t &m1, int64_t &m2)
@@ -823,6 +831,10 @@ struct Builder {
                 const int64_t q = n2 / r;
                 if (tr <= 1 || q < 2 || (c * q) % tr) continue;
                 if (q > dev.max_lds_len[plan.dtype] || !is_13smooth(q) || split_strided(q, r)) continue;
+                // a middle pass of half lines pays beyond 32 MiB only, and the three passes round more
+                // than two (3732480 points: 57.5 us and 2.24e-7, in two passes 54.5 us and 1.76e-7;
+                // 4478976: 66 and 101 us)
+                if (o * n * (int64_t)esz() <= ((int64_t)32 << 20) && !whole_lines(q, r)) continue;
                 n1 = c;
                 m1 = q;
                 m2 = r;

@@ -29,6 +29,8 @@ CASES = [
     (torch.complex128, 79, 824, 4.71e-16),
     # rows through the split exchange
     (torch.complex128, 260, 8192, 2.36e-16),
+    # two passes or three
+    (torch.complex64, 1, 3732480, 1.79e-7),
 ]
 
 
