@@ -95,7 +95,22 @@ template <typename V, int E> struct ColFft<V, E, 0> {
     }
 };
 
-template <typename Real, int E, int N, int... Rs>
+// The E elements of a column that a thread holds, T rows apart, at one 32-bit byte offset per thread: a
+// descriptor of the image and uniform offsets, or (BIG: images of 4 GiB and more) a descriptor of T rows
+// for each.
+template <typename V, bool BIG> struct ColumnView {
+    const V *base;
+    int64_t step; // elements
+    int64_t bytes;
+    __device__ __forceinline__ ColumnView(const void *p, int64_t first, int64_t h, int64_t w, int T)
+        : base(reinterpret_cast<const V *>(p) + first), step(T * w), bytes((BIG ? T : h) * w * (int64_t)sizeof(V)) {}
+    __device__ __forceinline__ BufView at(int i) const { return BufView(BIG ? base + i * step : base, (uint32_t)bytes); }
+    __device__ __forceinline__ uint32_t uniform(int i) const { return BIG ? 0 : i * (uint32_t)(step * (int64_t)sizeof(V)); }
+    __device__ __forceinline__ V load(int i, uint32_t off) const { return buf_load<V>(at(i), off, uniform(i)); }
+    __device__ __forceinline__ void store(int i, uint32_t off, V v) const { buf_store<V>(at(i), off, uniform(i), v); }
+};
+
+template <typename Real, int E, int N, bool BIG, int... Rs>
 __global__ void __launch_bounds__(max_block_threads(sizeof(Real) == 8, E)) afft_colconv(const ColConvArgs a)
 {
     using V = typename cplx_of<Real>::type;
@@ -108,18 +123,15 @@ __global__ void __launch_bounds__(max_block_threads(sizeof(Real) == 8, E)) afft_
     colconv_tile(tiles, a.B, b, ct);
     const int64_t j = ct * C + c;
     const bool active = j < a.w && b < a.B;
-    // an image is below 4 GiB (col_shape): one byte offset per thread, `step` bytes between its rows
-    const uint32_t bytes = (uint32_t)(a.h * a.w * (int64_t)sizeof(V)), step = (uint32_t)(T * a.w * (int64_t)sizeof(V));
-    const BufView d(reinterpret_cast<V *>(a.data) + b * a.h * a.w, bytes);
-    const BufView sp(reinterpret_cast<V *>(a.spec) + b * a.h * a.w, bytes);
-    const BufView Hc(reinterpret_cast<const V *>(a.H), bytes);
+    using View = ColumnView<V, BIG>;
+    const View d(a.data, b * a.h * a.w, a.h, a.w, T), sp(a.spec, b * a.h * a.w, a.h, a.w, T), Hc(a.H, 0, a.h, a.w, T);
     const uint32_t off = (uint32_t)((t * a.w + j) * (int64_t)sizeof(V));
     ColFft<V, E, N, Rs...> fft;
     fft.init(a, t);
     V reg[E];
     if (active) { // one branch around the whole batch of loads
 #pragma unroll
-        for (int i = 0; i < E; ++i) reg[i] = buf_load<V>(d, off, i * step);
+        for (int i = 0; i < E; ++i) reg[i] = d.load(i, off);
     } else {
 #pragma unroll
         for (int i = 0; i < E; ++i) reg[i] = c_make<V>(0, 0);
@@ -135,11 +147,11 @@ __global__ void __launch_bounds__(max_block_threads(sizeof(Real) == 8, E)) afft_
             V h[E4];
 #pragma unroll
             for (int i = 0; i < E4; ++i)
-                if (g + i < E) h[i] = buf_load<V>(Hc, off, (g + i) * step);
+                if (g + i < E) h[i] = Hc.load(g + i, off);
             if (a.spec) {
 #pragma unroll
                 for (int i = 0; i < E4; ++i)
-                    if (g + i < E) buf_store<V>(sp, off, (g + i) * step, reg[g + i]);
+                    if (g + i < E) sp.store(g + i, off, reg[g + i]);
             }
 #pragma unroll
             for (int i = 0; i < E4; ++i)
@@ -149,7 +161,7 @@ __global__ void __launch_bounds__(max_block_threads(sizeof(Real) == 8, E)) afft_
     fft.run(reg, lds + c, a, t);
     if (active) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) buf_store<V>(d, off, i * step, c_conj(reg[i]));
+        for (int i = 0; i < E; ++i) d.store(i, off, c_conj(reg[i]));
     }
 }
 
@@ -162,7 +174,7 @@ constexpr int vjp_block(bool f64) { return f64 ? 256 : 512; }
 // before the current image's inverse transform and its stores: loads and stores retire in order, so
 // loads behind the stores would wait for them too, and with one workgroup to a CU nothing else hides
 // either.
-template <typename Real, int E, int N, bool SPEC, int... Rs>
+template <typename Real, int E, int N, bool SPEC, bool BIG, int... Rs>
 __global__ void __launch_bounds__(vjp_block(sizeof(Real) == 8)) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 2 : 1, 8))) afft_colconv_vjp(const ColConvArgs a)
 {
     using V = typename cplx_of<Real>::type;
@@ -178,18 +190,18 @@ __global__ void __launch_bounds__(vjp_block(sizeof(Real) == 8)) __attribute__((a
     const int64_t per = (a.B + a.groups - 1) / a.groups;
     const int64_t b0 = g * per, b1 = (b0 + per < a.B) ? b0 + per : a.B;
     const int64_t image = a.h * a.w;
-    const uint32_t bytes = (uint32_t)(image * (int64_t)sizeof(V)), step = (uint32_t)(T * a.w * (int64_t)sizeof(V));
     const V *xs = reinterpret_cast<const V *>(a.other);
     V *gs = reinterpret_cast<V *>(a.data);
-    const BufView Hc(reinterpret_cast<const V *>(a.H), bytes);
+    using View = ColumnView<V, BIG>;
+    const View Hc(a.H, 0, a.h, a.w, T);
     const uint32_t off = (uint32_t)((t * a.w + j) * (int64_t)sizeof(V));
     ColFft<V, E, N, Rs...> fft;
     fft.init(a, t);
     auto load = [&](V (&r)[E], const V *p) {
-        const BufView v(p, bytes);
+        const View v(p, 0, a.h, a.w, T);
         if (active) { // one branch around the whole batch
 #pragma unroll
-            for (int i = 0; i < E; ++i) r[i] = buf_load<V>(v, off, i * step);
+            for (int i = 0; i < E; ++i) r[i] = v.load(i, off);
             __builtin_amdgcn_sched_barrier(0);
         } else {
 #pragma unroll
@@ -216,7 +228,7 @@ __global__ void __launch_bounds__(vjp_block(sizeof(Real) == 8)) __attribute__((a
         if (active) {
             V h[E];
 #pragma unroll
-            for (int i = 0; i < E; ++i) h[i] = buf_load<V>(Hc, off, i * step);
+            for (int i = 0; i < E; ++i) h[i] = Hc.load(i, off);
             __builtin_amdgcn_sched_barrier(0); // every filter load in flight before the first is used
 #pragma unroll
             for (int i = 0; i < E; ++i) {
@@ -227,9 +239,9 @@ __global__ void __launch_bounds__(vjp_block(sizeof(Real) == 8)) __attribute__((a
         if (b + 1 < b1) load(X, (SPEC ? (const V *)gs : xs) + (b + 1) * image);
         fft.run(G, lds + c, a, tl);
         if (active) {
-            const BufView v(gs + b * image, bytes);
+            const View v(gs, b * image, a.h, a.w, T);
 #pragma unroll
-            for (int i = 0; i < E; ++i) buf_store<V>(v, off, i * step, c_conj(G[i]));
+            for (int i = 0; i < E; ++i) v.store(i, off, c_conj(G[i]));
         }
         if constexpr (SPEC) {
 #pragma unroll
@@ -237,9 +249,9 @@ __global__ void __launch_bounds__(vjp_block(sizeof(Real) == 8)) __attribute__((a
         }
     }
     if (active) {
-        const BufView v(reinterpret_cast<V *>(a.partial) + g * image, bytes);
+        const View v(a.partial, g * image, a.h, a.w, T);
 #pragma unroll
-        for (int i = 0; i < E; ++i) buf_store<V>(v, off, i * step, acc[i]);
+        for (int i = 0; i < E; ++i) v.store(i, off, acc[i]);
     }
 }
 
@@ -309,17 +321,23 @@ int residual_rows(const Plan &rp, int dtype, const void *y, const void *t, doubl
 
 #define AFFT_SPEC_E(X) X(1) X(2) X(3) X(4) X(5) X(6) X(8) X(9) X(10) X(12) X(15) X(16)
 
-template <typename Real> const void *colconv_fn(bool vjp, bool spec, int E, int64_t h)
+template <typename Real> const void *colconv_fn(bool vjp, bool spec, int E, int64_t h, bool big)
 {
 #define AFFT_COLCONV(EV, H, ...)                                                                 \
-    return !vjp ? reinterpret_cast<const void *>(afft_colconv<Real, EV, H, ##__VA_ARGS__>)       \
-         : spec ? reinterpret_cast<const void *>(afft_colconv_vjp<Real, EV, H, true, ##__VA_ARGS__>) \
-                : reinterpret_cast<const void *>(afft_colconv_vjp<Real, EV, H, false, ##__VA_ARGS__>)
+    return !vjp ? reinterpret_cast<const void *>(afft_colconv<Real, EV, H, __VA_ARGS__>)         \
+         : spec ? reinterpret_cast<const void *>(afft_colconv_vjp<Real, EV, H, true, __VA_ARGS__>) \
+                : reinterpret_cast<const void *>(afft_colconv_vjp<Real, EV, H, false, __VA_ARGS__>)
     // compile-time transforms for the common heights (the radices of the row kernels)
-    if (h == 256 && E == 16) AFFT_COLCONV(16, 256, 16, 16);
-    if (h == 512 && E == 16) AFFT_COLCONV(16, 512, 16, 16, 2);
+    if (h == 256 && E == 16) {
+        if (big) AFFT_COLCONV(16, 256, true, 16, 16);
+        AFFT_COLCONV(16, 256, false, 16, 16);
+    }
+    if (h == 512 && E == 16) {
+        if (big) AFFT_COLCONV(16, 512, true, 16, 16, 2);
+        AFFT_COLCONV(16, 512, false, 16, 16, 2);
+    }
     switch (E) {
-#define X(EV) case EV: AFFT_COLCONV(EV, 0);
+#define X(EV) case EV: if (big) AFFT_COLCONV(EV, 0, true); AFFT_COLCONV(EV, 0, false);
         AFFT_SPEC_E(X)
 #undef X
 #undef AFFT_COLCONV
@@ -327,11 +345,14 @@ template <typename Real> const void *colconv_fn(bool vjp, bool spec, int E, int6
     }
 }
 
+// whether the byte offsets of an image exceed 32 bits
+bool big_image(int dtype, int64_t h, int64_t w) { return h * w >= ((int64_t)1 << 32) / (dtype == AFFT_C64 ? 8 : 16); }
+
 template <typename Real>
 hipError_t launch_colconv(bool vjp, int E, const ColConvArgs &a, int block, int64_t grid, size_t lds,
                           hipStream_t s)
 {
-    const void *fn = colconv_fn<Real>(vjp, a.other_is_spec, E, a.h);
+    const void *fn = colconv_fn<Real>(vjp, a.other_is_spec, E, a.h, big_image(sizeof(Real) == 8, a.h, a.w));
     if (!fn) return hipErrorInvalidValue;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -350,8 +371,6 @@ struct ColShape {
 bool col_shape(int dtype, int64_t h, int64_t w, ColShape &cs, bool vjp)
 {
     if (h > 16384 || !is_5smooth(h)) return false;
-    // the column kernels address an image with 32-bit byte offsets
-    if (h * w >= ((int64_t)1 << 32) / (dtype == AFFT_C64 ? 8 : 16)) return false;
     if (!choose_layout(h, dtype, cs.L, 16, vjp ? vjp_block(dtype == AFFT_C128) : -1)) return false;
     const int T = (int)(h / cs.L.E);
     const int maxb = vjp ? vjp_block(dtype == AFFT_C128) : max_block_threads(dtype == AFFT_C128, cs.L.E);
@@ -361,6 +380,10 @@ bool col_shape(int dtype, int64_t h, int64_t w, ColShape &cs, bool vjp)
     if (cs.C * T > maxb) return false;
     cs.block = cs.C * T;
     cs.lds = cs.L.npass > 1 ? (size_t)cs.C * lds_padded_len((int)h) * esz : 0;
+    // images of 4 GiB and more: the column kernels address T rows at a time with 32-bit byte offsets, and
+    // pay where their tiles read whole lines (512 x 2^20 Complex Float fused 12.5 and 18.0 ms, forward and
+    // VJP, unfused 16.9 and 21.5 ms; 4096 x 131072, 32-byte tiles, 19.5 and 29.4 against 19.6 and 24.3 ms)
+    if (big_image(dtype, h, w) && ((size_t)cs.C * esz < 128 || (size_t)T * w * esz >= ((size_t)1 << 32))) return false;
     return cs.lds <= 160 * 1024;
 }
 

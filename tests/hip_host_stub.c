@@ -5,11 +5,12 @@
 #include <hip/hip_runtime_api.h>
 #include <stdlib.h>
 
-static unsigned long long most_groups, most_threads;
+static unsigned long long most_groups, most_threads, launches;
 
 unsigned long long stub_most_groups(void) { return most_groups; }
 unsigned long long stub_most_threads(void) { return most_threads; }
-void stub_reset(void) { most_groups = most_threads = 0; }
+unsigned long long stub_launches(void) { return launches; }
+void stub_reset(void) { most_groups = most_threads = launches = 0; }
 
 hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
@@ -80,6 +81,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, si
 {
     (void)f; (void)args; (void)lds; (void)s;
     const unsigned long long g = (unsigned long long)grid.x * grid.y * grid.z;
+    ++launches;
     if (g > most_groups) most_groups = g;
     if (g * block.x > most_threads) most_threads = g * block.x;
     return hipSuccess;

@@ -17,7 +17,7 @@ L = importlib.util.module_from_spec(spec)
 spec.loader.exec_module(L)
 lib = L.lib()
 stub = ctypes.CDLL(None)
-stub.stub_most_groups.restype = stub.stub_most_threads.restype = ctypes.c_ulonglong
+stub.stub_most_groups.restype = stub.stub_most_threads.restype = stub.stub_launches.restype = ctypes.c_ulonglong
 
 def plan(dtype, *ext, axes=L.AXES_INNERMOST):
     h = ctypes.c_void_p()
@@ -88,4 +88,22 @@ for dtype in (L.C64, L.C128):
         assert 1 <= groups <= max(1024, shape[0] // 256 + 1), (dtype, shape, groups)
         assert threads < 1 << 32
         lib.afft_plan_destroy(h)
+""")
+
+
+def test_spectral_images_of_4_gib_stay_fused(stub):
+    """The fused spectral convolution runs the row transforms twice and one launch over the columns,
+    also for images of 4 GiB and more whose column tiles read whole lines (the unfused one transforms the
+    columns on their own)."""
+    run_child(stub, """
+for dtype, h, w in ((L.C64, 32, 1 << 20), (L.C64, 32, 1 << 24), (L.C64, 512, 1 << 21), (L.C128, 16, 1 << 24)):
+    st, h1 = plan(dtype, h, w)
+    assert st == 0
+    stub.stub_reset()
+    assert lib.afft_exec(h1, -1, 256, 256, 1.0, None) == 0
+    rows = stub.stub_launches()
+    assert lib.afft_spectral_conv_fwd(dtype, 1, h, w, 256, 512, 768, None) == 0  # (makes the tables)
+    stub.stub_reset()
+    assert lib.afft_spectral_conv_fwd(dtype, 1, h, w, 256, 512, 768, None) == 0
+    assert stub.stub_launches() == 2 * rows + 1, (dtype, h, w, rows, stub.stub_launches())
 """)
