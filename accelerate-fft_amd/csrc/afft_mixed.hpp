@@ -1,4 +1,4 @@
-// afft_mixed.hpp -- descriptors of the mixed-radix kernel (afft_mixed.hip): transforms of any length
+// afft_mixed.hpp -- descriptors of the mixed-radix kernel (afft_mixed_kernel.hpp): transforms of any length
 // whose prime factors are at most 13 (31 where the length fits a workgroup), and chirp-z transforms of
 // the others, for contiguous rows and for strided axes.
 #pragma once
@@ -17,8 +17,8 @@ constexpr int kMixMaxRadix = 16;
 // of it a thread: a prime p costs about p operations an element in one pass, a chirp-z transform
 // 130 ... 200 in five (its E; the other radices as with 16 elements).  128 MiB of Complex Float rows of 31:
 // 102 -> 60 us, of 289 138 -> 55 us, of 16337 563 -> 113 us; Complex Double rows of 4913 609 -> 92 us.
-// Instances of their own, since a butterfly of 31 takes the registers of four waves a SIMD (one of 23
-// Complex Double those of two; of 29 it would spill).
+// Instances of their own, since a butterfly of 31 takes the registers of four waves a SIMD (the strided form
+// spills 40 bytes a lane), one of 23 Complex Double those of two.
 constexpr int kMixWide = 31;
 constexpr int mixed_wide_radix(int dtype) { return dtype == 0 ? 31 : 23; }
 
@@ -39,9 +39,12 @@ struct MixPass {
     int rpad, rstep, wblock;
 };
 
-// Waves per SIMD the registers of a kernel must allow.  Where more would spill the strided kernels
-// keep what the compiler needs: forced to 7 (from 82 registers to 72, 15 spilled) the Complex Float
-// tiles of 100 and 224 points took 53 us instead of 42 on 128 MiB.
+// Waves per SIMD the registers of a kernel must allow, and that the planner counts as resident.  Where
+// more would spill the strided kernels keep what the compiler needs: forced to 7 (from 82 registers to
+// 72, 15 spilled) the Complex Float tiles of 100 and 224 points took 53 us instead of 42 on 128 MiB.  (The
+// Complex Float kMixWide kernels have 4 from their launch bound; counted as 4 the planner takes slower
+// tiles for a few lengths and faster ones for none: 2^23 elements in rows of 58 65 -> 97 us, of 19 26 -> 31
+// us.)
 __host__ __device__ constexpr int mixed_waves(bool f64, int E, bool rows, bool chirpz)
 {
     if (E == kMixWide) return f64 ? 2 : 3;
