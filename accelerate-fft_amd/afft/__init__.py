@@ -170,8 +170,9 @@ def vjp(op, mode, gy):
 
 
 def describe(n, dtype=torch.complex64):
-    """Host-only: (radices, elements per thread, Bluestein length or 0) of the
-    single-workgroup layout for length n; raises AfftError beyond the LDS limit."""
+    """Host-only: (radices, elements per thread, Bluestein length or 0) of the pass-table layout for length n,
+    which the columns of spectral convolutions run (afft_describe in include/afft.h; other transforms choose
+    their radices per plan); raises AfftError beyond the LDS limit."""
     code = L.C64 if dtype == torch.complex64 else L.C128
     rad = (ctypes.c_int * 32)()
     npass, E = ctypes.c_int(), ctypes.c_int()

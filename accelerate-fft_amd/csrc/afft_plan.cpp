@@ -677,8 +677,8 @@ struct Builder {
     // round of 24576 Complex Float takes 21 ... 29 us, two passes 18 us and 24 us more per 256
     // rows: 42.7 -> 28.7 us for 256 rows, 142 -> 112 us for 1024, but 47 -> 50 us for 300 and 19.8 -> 21 us
     // for 16; 32768: 54 -> 39 us for 256, 18.6 -> 27 us for 16; Complex Double 16384: 66 -> 37 us.
-    // Complex Double rows of those lengths keep their two passes as one axis of several: plans of two
-    // split axes, with the data moving between output and work buffer, are to stay what they are.
+    // Complex Double rows of those lengths keep their two passes as one axis of several, where the single
+    // pass was not measured: the launches of 2048 x 16384, two split axes, are fixed by a test.
     bool split_rows_idle(int64_t n, int64_t o)
     {
         if (n <= (plan.dtype == AFFT_C64 ? 20480 : 10240)) return false;

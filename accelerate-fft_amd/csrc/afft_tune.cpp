@@ -115,7 +115,7 @@ bool plausible(int kind, int dtype, int64_t n, int value)
         return C >= 1 && C <= 64 && (C & (C - 1)) == 0 && E >= 1 && n % E == 0;
     }
     case kTuneRegcol: return (value == 1 || value == 2 || value == 4) && regcol_supported(dtype, n);
-    case kTuneRagged: return value >= 0 && value <= 32; // 0: whole workgroups, 1: half of them
+    case kTuneRagged: return value >= 0 && value <= 32; // 0: whole workgroups, 1: half of them (others: no candidate any more)
     case kTuneRaggedSplit: return value >= 0;          // elements below which a class goes aside
     default: return false;
     }

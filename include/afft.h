@@ -190,10 +190,15 @@ int afft_plan_info(const afft_plan *plan, int *launches, int64_t *device_bytes);
 
 /* ---- host-only planning (no device needed) ---------------------------------------------- */
 
-/* Describe how a single-workgroup LDS transform of length n would be laid out: the radix of each
- * Stockham pass (at most max_passes written), elements per thread, and the Bluestein padded
- * length (0 when n is 5-smooth).  Returns AFFT_ERROR_UNSUPPORTED_SIZE when n is beyond the
- * single-workgroup limit for the dtype (the multi-pass four-step path then applies). */
+/* Describe the pass-table layout of a transform of length n held by one workgroup: the radix of each
+ * Stockham pass (at most max_passes written) and the elements per thread.  The columns of spectral
+ * convolutions (afft_spectral_conv_*, heights n that are products of 2, 3 and 5) run these passes; other
+ * transforms run compiled layouts (rows, some strided lengths) or choose mixed radices per plan, which this
+ * does not report.  For other n the layout is that of *bluestein_len, the padded length of a chirp-z
+ * transform in several launches (0 when n is 5-smooth); chirp-z transforms held by one workgroup may take
+ * another.  Returns AFFT_ERROR_UNSUPPORTED_SIZE when the length is beyond one workgroup for the dtype, and
+ * for the few 5-smooth lengths without a layout, which plans refuse too (12800 in Complex Float, 8000 in
+ * Complex Double, ...). */
 int afft_describe(int64_t n, int dtype, int *radices, int max_passes, int *n_passes,
                   int *elems_per_thread, int64_t *bluestein_len);
 
