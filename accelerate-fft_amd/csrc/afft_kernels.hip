@@ -10,6 +10,8 @@
 // exchanged through LDS.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "afft_device.hpp"
 #include "afft_internal.hpp"
 #include "afft_mixed.hpp"
@@ -172,15 +174,22 @@ __global__ void afft_gen_pass_twiddles(typename cplx_of<Real>::type *out, const 
     }
 }
 
+struct MixTables { // of the passes after the first
+    int npass;
+    MixPass pass[kMixMaxPasses];
+};
+
 template <typename Real>
-__global__ void afft_gen_mixed_twiddles(typename cplx_of<Real>::type *out, int Ns, int R)
+__global__ void afft_gen_mixed_twiddles(typename cplx_of<Real>::type *out, const MixTables t)
 {
     using V = typename cplx_of<Real>::type;
-    const int count = mixed_twiddle_elems(sizeof(Real) == 8, Ns, R);
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (R + 1) * Ns; i += gridDim.x * blockDim.x) {
-        const int r = i / Ns + 1, k = i % Ns, at = mixed_twiddle_at(sizeof(Real) == 8, Ns, r, k);
-        const double2 w = unit_root(r == R ? 0 : r * k, Ns * R); // (r k < Ns R < 2^31; r = R: the spare halves)
-        if (at < count) out[at] = c_make<V>((Real)w.x, (Real)w.y);
+    for (int p = 1; p < t.npass; ++p) {
+        const int Ns = t.pass[p].Ns, R = t.pass[p].R, count = mixed_twiddle_elems(sizeof(Real) == 8, Ns, R);
+        for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < R * Ns; i += gridDim.x * blockDim.x) {
+            const int r = i / Ns + 1, k = i % Ns, at = mixed_twiddle_at(sizeof(Real) == 8, Ns, r, k);
+            const double2 w = unit_root(r == R ? 0 : r * k, Ns * R); // (r = R: the spare halves)
+            if (at < count) out[t.pass[p].toff + at] = c_make<V>((Real)w.x, (Real)w.y);
+        }
     }
 }
 
@@ -325,14 +334,14 @@ hipError_t gen_pass_twiddles(int dtype, void *out, const PassTable &pt, hipStrea
 
 hipError_t gen_mixed_twiddles(int dtype, void *out, const MixArgs &a, hipStream_t s)
 {
-    for (int i = 1; i < a.npass; ++i) {
-        const MixPass &p = a.pass[i];
-        const int64_t g = gs_grid((int64_t)p.Ns * (p.R + 1));
-        if (dtype == 0)
-            hipLaunchKernelGGL(afft_gen_mixed_twiddles<float>, dim3(g), dim3(256), 0, s, (float2 *)out + p.toff, p.Ns, p.R);
-        else
-            hipLaunchKernelGGL(afft_gen_mixed_twiddles<double>, dim3(g), dim3(256), 0, s, (double2 *)out + p.toff, p.Ns, p.R);
-    }
+    MixTables t;
+    t.npass = a.npass;
+    std::copy(a.pass, a.pass + a.npass, t.pass);
+    const int64_t g = gs_grid(a.n);
+    if (dtype == 0)
+        hipLaunchKernelGGL(afft_gen_mixed_twiddles<float>, dim3(g), dim3(256), 0, s, (float2 *)out, t);
+    else
+        hipLaunchKernelGGL(afft_gen_mixed_twiddles<double>, dim3(g), dim3(256), 0, s, (double2 *)out, t);
     return hipGetLastError();
 }
 
