@@ -139,11 +139,10 @@ extern "C" int afft_fft_centred(int mode, int dtype, int rank, const int64_t *ex
     if (!valid_which(pre) || !valid_which(post)) return AFFT_ERROR_INVALID_VALUE;
     int st = check_reorder_shape(dtype, rank, extents);
     if (st) return st;
-    int64_t total = 1, halves = 0;
+    int64_t total = 1;
     bool all_even = true;
     for (int d = 0; d < rank; ++d) {
         total *= extents[d];
-        halves += extents[d] / 2;
         all_even = all_even && (extents[d] % 2 == 0);
     }
     if (total == 0) return AFFT_SUCCESS;
@@ -157,8 +156,6 @@ extern "C" int afft_fft_centred(int mode, int dtype, int rank, const int64_t *ex
     bool load_sign = pre == AFFT_CENTRE, store_sign = post == AFFT_CENTRE;
     bool roll_pre = pre == AFFT_SHIFT || pre == AFFT_ISHIFT;
     bool roll_post = post == AFFT_SHIFT || post == AFFT_ISHIFT;
-    // the roll of the output moves the sign that stands for a roll of the input by n / 2 along every axis
-    const bool negate = all_even && roll_pre && roll_post && halves % 2;
     if (roll_post && all_even) {
         load_sign = !load_sign;
         roll_post = false;
@@ -184,7 +181,7 @@ extern "C" int afft_fft_centred(int mode, int dtype, int rank, const int64_t *ex
     }
     if (roll_post) dst = tmp; // with roll_pre too: the transform runs in place on the temporary
     const int dir = mode == AFFT_FORWARD ? -1 : 1;
-    const double scale = (mode == AFFT_INVERSE ? 1.0 / (double)total : 1.0) * (negate ? -1.0 : 1.0);
+    const double scale = mode == AFFT_INVERSE ? 1.0 / (double)total : 1.0;
     if (!st) st = exec_plan(*p, dir, src, dst, scale, s, nullptr, nullptr, load_sign ? &sg : nullptr,
                             store_sign ? &sg : nullptr);
     if (!st && roll_post) {
