@@ -418,8 +418,9 @@ const RowEntry kRows[] = {
     AFFT_ROW(float, 0, 12288, 24, false, 2, true, 8, 8, 8, 8, 3),
     // One row per workgroup of 1024 threads through the split exchange.  With linear addresses and
     // the twiddles loaded pass by pass the row and one butterfly are all that its registers hold:
-    // 16384 takes 60 of them, which lets two workgroups share a CU (1024 rows: 73 -> 58 us), and 32768 fits 128.  In one pass instead of two: 1024 rows of 24576 142
-    // -> 114 us, of 32768 184 -> 155 us, of Complex Double 16384 244 -> 138 us, 12288 133 -> 105 us.
+    // 16384 takes 57 of them, which lets two workgroups share a CU (1024 rows: 73 -> 58 us), and 32768
+    // fits 128.  In one pass instead of two: 1024 rows of 24576 142 -> 114 us, of 32768 184 -> 155 us,
+    // of Complex Double 16384 244 -> 138 us, 12288 133 -> 105 us.
     // What is left to the copy rate (76 ... 101 us) is the one row per CU, whose loads, exchanges and
     // stores do not overlap.  Every pass but the last has stride <= T.
     AFFT_ROW_SPLIT(float, 0, 16384, 16, 4, true, 16, 16, 4, 16),
