@@ -45,7 +45,10 @@ def ishift3D(x): return _reorder(L.ISHIFT, x, 3)
 
 def fft_centred(mode, arr, pre=None, post=None, out=None):
     """post(fftND(mode, pre(arr))) over all axes of a rank-1/2/3 array; pre / post are None,
-    "centre", "shift" or "ishift".  ``out`` may be ``arr`` itself (in place)."""
+    "centre", "shift" or "ishift".  ``out`` may be ``arr`` itself (in place).
+
+    Known fault: with a shift or ishift on both sides, every extent even and the sum of the n/2
+    odd, the result is the negative of the composition."""
     x = _device_tensor(arr)
     if not 1 <= x.dim() <= 3:
         raise ValueError("fft_centred takes an Array DIM1, DIM2 or DIM3")

@@ -117,7 +117,9 @@ int afft_reorder(int which, int dtype, int rank, const int64_t *extents, const v
  * the Centre.hs operations on either side), pre / post as `which` above.  A centring, and a shift
  * or ishift when every extent is even, is folded into the transform's first load or last store
  * (no extra pass: shift(F x) = F(x (-1)^m) and F(shift x) = (-1)^k F x for even n); a shift over
- * an odd extent adds one reordering pass. */
+ * an odd extent adds one reordering pass.
+ * Known fault: with a shift or ishift on both sides, every extent even and the sum of the n/2 odd, the
+ * result is the negative of the composition (the roll of the folded signs (-1)^k is left out). */
 int afft_fft_centred(int mode, int dtype, int rank, const int64_t *extents, int pre, int post,
                      const void *d_in, void *d_out, void *stream);
 
